@@ -3,13 +3,18 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+import time
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libksq.so")
 
-SOURCES = ["ksq_api.hip", "ksq_repack.hip", "ksq_w4a16_stream.hip", "ksq_w4a16_kstat.hip", "ksq_w4a16_astream.hip", "ksq_w4a16_prefill.hip", "ksq_fp8.hip", "ksq_fp8_kstat.hip", "ksq_fp8_prefill.hip", "ksq_fp8_mid.hip"]
+# slowest to compile first: they start first (run_compilers)
+SOURCES = ["ksq_w4a16_prefill_f16.hip", "ksq_w4a16_prefill_bf16.hip", "ksq_w4a16_stream.hip", "ksq_w4a16_kstat.hip",
+           "ksq_fp8_kstat.hip", "ksq_w4a16_astream.hip", "ksq_fp8.hip", "ksq_fp8_prefill.hip", "ksq_fp8_mid.hip",
+           "ksq_repack.hip", "ksq_w4a16_prefill.hip", "ksq_api.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -52,23 +57,46 @@ def hipcc():
     return exe
 
 
-def build_library(verbose=False, jobs=5):
+def run_compilers(commands, done, jobs=None):
+    """commands: (source name, command line).  At most `jobs` at a time, each started as soon as another ends;
+    done(name, exit status, output) is called as they end, and every one that ended is named on stderr."""
+    jobs = jobs or max(1, min(16, int(os.environ.get("MAX_JOBS", "0")) or os.cpu_count() or 1))
+    waiting, running = list(commands), []
+    try:
+        while waiting or running:
+            while waiting and len(running) < jobs:
+                name, cmd = waiting.pop(0)
+                log = tempfile.TemporaryFile(mode="w+")
+                running.append((name, subprocess.Popen(cmd, stdout=log, stderr=subprocess.STDOUT), log, time.time()))
+            time.sleep(0.05)
+            for item in [r for r in running if r[1].poll() is not None]:
+                running.remove(item)
+                name, p, log, t0 = item
+                log.seek(0)
+                print(f"[build] {name} {time.time() - t0:.0f} s", file=sys.stderr, flush=True)
+                done(name, p.returncode, log.read())
+                log.close()
+    finally:
+        for _, p, log, _ in running:  # another one failed
+            p.kill()
+            p.wait()
+            log.close()
+
+
+def build_library(verbose=False, jobs=None):
     """Compile every HIP source to an object (in parallel) and link libksq.so next to this file."""
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     cc = hipcc()
-    procs = []
-    objs = []
+    objs, commands = [], []
     for src in SOURCES:
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
         objs.append(obj)
         cmd = [cc, *HIPCC_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
-        procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
-        if len(procs) >= jobs:
-            _drain(procs)
-    _drain(procs)
+        commands.append((src, cmd))
+    run_compilers(commands, _compiled, jobs)
     link = [cc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
     subprocess.check_call(link)
     return LIB
@@ -95,25 +123,23 @@ def build_layer_driver():
     return out
 
 
-def _drain(procs):
-    while procs:
-        src, p = procs.pop(0)
-        out, _ = p.communicate()
-        remarks, lines, skip = [], [], 0
-        for ln in out.splitlines():
-            if "-Rpass-analysis=kernel-resource-usage" in ln:
-                remarks.append(ln)
-                skip = 2  # the source line and the caret that follow a remark
-            elif skip and ln.lstrip()[:1] in "0123456789|":
-                skip -= 1
-            elif "packed-fp32-ops" not in ln and "remarks generated" not in ln:
-                skip = 0
-                lines.append(ln)
-        if p.returncode != 0:
-            raise RuntimeError(f"hipcc failed on {src}:\n" + "\n".join(lines))
-        check_scratch(src, remarks)
-        if lines:
-            print("\n".join(lines), file=sys.stderr)
+def _compiled(src, status, out):
+    """One source file's compiler output: its messages without the resource remarks, which check_scratch reads."""
+    remarks, lines, skip = [], [], 0
+    for ln in out.splitlines():
+        if "-Rpass-analysis=kernel-resource-usage" in ln:
+            remarks.append(ln)
+            skip = 2  # the source line and the caret that follow a remark
+        elif skip and ln.lstrip()[:1] in "0123456789|":
+            skip -= 1
+        elif "packed-fp32-ops" not in ln and "remarks generated" not in ln and "In file included from" not in ln:
+            skip = 0
+            lines.append(ln)
+    if status != 0:
+        raise RuntimeError(f"hipcc failed on {src}:\n" + "\n".join(lines))
+    check_scratch(src, remarks)
+    if lines:
+        print("\n".join(lines), file=sys.stderr)
 
 
 if __name__ == "__main__":

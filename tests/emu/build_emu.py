@@ -7,7 +7,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
 sys.path.insert(0, ROOT)
-from ksanallm_amd.build import CSRC, SOURCES  # noqa: E402
+from ksanallm_amd.build import CSRC, SOURCES, run_compilers  # noqa: E402
 
 LIB = os.path.join(HERE, "libksq_emu.so")
 LIB_ASAN = os.path.join(HERE, "libksq_emu_asan.so")
@@ -24,42 +24,49 @@ def flags(asan):
     f = ["-x", "c++", "-std=c++17", "-O1", "-g1", "-fPIC", "-march=x86-64-v3", "-pthread",
          "-I" + os.path.join(HERE, "include"), "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
          "-Wno-unknown-attributes", "-Wno-ignored-attributes", "-Wno-unused-function", "-Wno-pass-failed",
-         "-Wno-unknown-pragmas"]
+         "-Wno-unknown-pragmas",
+         # the kernels' "#pragma unroll" ignored: nothing here needs the loops unrolled, and unrolled they take three times as
+         # long to compile (five times with the sanitizer)
+         "-mllvm", "-pragma-unroll-threshold=0"]
     if asan:
         f += ["-fsanitize=address", "-fno-omit-frame-pointer"]
     return f
 
 
-def build(asan=False, jobs=8, verbose=False):
+def build(asan=False, jobs=None, verbose=False):
     cc = clangxx()
     objdir = os.path.join(HERE, "build_asan" if asan else "build")
     os.makedirs(objdir, exist_ok=True)
     srcs = [os.path.join(CSRC, s) for s in SOURCES] + [os.path.join(HERE, "emu_runtime.cpp")]
-    objs, procs = [], []
+    objs, commands = [], []
 
-    def drain():
-        while procs:
-            name, p = procs.pop(0)
-            out, _ = p.communicate()
-            if p.returncode != 0:
-                raise RuntimeError(f"host build of {name} failed:\n{out[-6000:]}")
-            if verbose and out.strip():
-                print(out, file=sys.stderr)
+    def done(name, status, out):
+        if status != 0:
+            raise RuntimeError(f"host build of {name} failed:\n{out[-6000:]}")
+        if verbose and out.strip():
+            print(out, file=sys.stderr)
 
     for src in srcs:
         obj = os.path.join(objdir, os.path.basename(src).rsplit(".", 1)[0] + ".o")
         objs.append(obj)
-        cmd = [cc, *flags(asan), "-c", src, "-o", obj]
-        procs.append((os.path.basename(src), subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
-        if len(procs) >= jobs:
-            drain()
-    drain()
+        commands.append((os.path.basename(src), [cc, *flags(asan), "-c", src, "-o", obj]))
+    run_compilers(commands, done, jobs)
     out = LIB_ASAN if asan else LIB
     link = [cc, "-shared", "-pthread", "-o", out, *objs]
     if asan:
         link += ["-fsanitize=address", "-shared-libasan"]
     subprocess.check_call(link)
     return out
+
+
+def up_to_date(lib):
+    """Whether `lib` is there and newer than everything it is built from."""
+    if not os.path.exists(lib):
+        return False
+    files = [os.path.join(HERE, "emu_runtime.cpp"), os.path.join(HERE, "include", "hip", "hip_runtime.h"), __file__]
+    for d in (CSRC, os.path.join(ROOT, "include")):
+        files += [os.path.join(d, f) for f in os.listdir(d) if f.endswith((".h", ".hip"))]
+    return os.path.getmtime(lib) >= max(os.path.getmtime(f) for f in files)
 
 
 def build_layer_driver():

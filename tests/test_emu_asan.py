@@ -24,7 +24,7 @@ def test_parity_slice_under_address_sanitizer():
         pytest.skip("the sanitizer runtime of the ROCm clang is not installed")
     from tests.emu import build_emu
 
-    if not os.path.exists(build_emu.LIB_ASAN):
+    if not build_emu.up_to_date(build_emu.LIB_ASAN):
         build_emu.build(asan=True)
     env = dict(os.environ, KSQ_EMU_ASAN="1", KSQ_EMU_THREADS="1",
                LD_PRELOAD=rt + (":" + os.environ["LD_PRELOAD"] if os.environ.get("LD_PRELOAD") else ""),
