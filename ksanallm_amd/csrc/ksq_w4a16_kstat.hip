@@ -9,10 +9,13 @@
 // tile per wave.  Because k is covered inside the workgroup, narrow N needs no split across workgroups; only K
 // beyond waves x TPW tiles is split over grid.y and finished by the last-arriving workgroup through the workspace.
 //
-// Arithmetic: biased nibbles by bit operations, fp32 group sums scaled by s[g,n]; bias and zero point are taken out once
-// per column tile by an fp32 MFMA over the groups (GroupCorrection), or, with few groups per wave, from the start value
-// of every group's accumulator.  A correction MFMA of -(bias + z) per 32 k, as in the streaming kernel, doubles the
-// matrix instructions: Llama-3-70B gate_up at M = 32 69.4 us against 64.3, M = 16 44.9 against 42.0.
+// Arithmetic: biased nibbles by bit operations, fp32 group sums scaled by s[g,n].  What bias and zero point owe comes out of
+// every group's own sum, before its scale: as the value that the sum starts from, made of the activations' row sums (in registers
+// with few groups per wave, otherwise by one matrix instruction, GroupStart), or by a correction MFMA of -(bias + z) per 32 k, as
+// in the streaming kernel, which doubles the matrix instructions: Llama-3-70B gate_up at M = 27 77 us against 58.7, M = 16 48
+// against 42.8, 4096 x 22016 at M = 32 17.1 against 15.4.  (All groups at once, as an fp32 product of row sums and scaled columns,
+// is 1 to 5 % faster still, but a sum then carries its bias through all groups of a wave -- up to 14 % of the fp16 outputs were not
+// the rounded exact result, now 0.1 to 0.3 %, with the correction 1.6 to 3.4 % -- and overflows where the result does not.)
 #include <cstdlib>
 
 #include "ksq_internal.h"
@@ -46,7 +49,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
   using O = Ops<T>;
   constexpr int DPG = 4 / GPT;
   constexpr int D = NB * TPW;  // ring depth = one batch
-  constexpr bool kRowSums = MT == 1 && TPW * GPT <= 2 && D <= 4;  // see the prologue
   constexpr bool kSumAtEnd = MT > 1;  // of K splits, see splitk_finish_workgroup
   static_assert(NB * MT * NW <= 64 && NB * MT <= NW && NW % (NB * MT) == 0, "reduction: two buffers of <= 64 KiB");
   __shared__ f32x4 red[2 * NB * MT * NW * 64];
@@ -87,25 +89,22 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
   // The scale/zero words of one batch -- NB column tiles x the wave's TPW * GPT groups x 16 columns -- are fetched
   // with one word per lane: the words of one column tile are contiguous (its groups follow each other), so SZR
   // instructions cover the batch instead of one instruction per (column tile, group).  Flat word f = 64 r + lane
-  // belongs to column tile f / (16 GP), group (f / 16) % GP, column f % 16, with GP = the groups rounded up so that a
-  // column tile never straddles an instruction: the words of an instruction are then the column operand of the
-  // correction (GroupCorrection) for one column tile, or for 4 / GP of them.  The memory pipeline takes about as long
-  // for a one-word-per-lane instruction as for a weight tile, so the number of instructions matters.
-  constexpr int GW = TPW * GPT;  // groups per column tile that this wave needs
-  constexpr int GP = GW <= 1 ? 1 : GW <= 2 ? 2 : (GW + 3) / 4 * 4;
-  constexpr int SZR = (NB * GP * 16 + 63) / 64;  // instructions per batch
-  constexpr int CG = (GP + 3) / 4;               // correction instructions per column tile, row tile and term
-  // fp16 with six or eight groups: the nibbles all with bias 1024 (two more shifts per eight), whose correction has one
-  // term instead of two -- with two the registers of sixteen waves do not hold it (groups of 64, K = 6528, one token:
-  // spilled 35 us, so 20)
-  constexpr bool kUniform = !__is_same(T, _Float16) || (MT == 1 && GW > 4);
-  using Correction = GroupCorrection<T, kUniform>;
-  constexpr int kTerms = Correction::kTerms;
+  // belongs to column tile f / (16 GW), group (f / 16) % GW, column f % 16.  The memory pipeline takes about as long
+  // for a one-word-per-lane instruction as for a weight tile, so this matters.
+  constexpr int GW = TPW * GPT;                  // groups per column tile that this wave needs
+  constexpr int SZR = (NB * GW * 16 + 63) / 64;  // instructions per batch
+  // How bias and zero point leave the sums: row sums in registers where there is room for them (4096 x 22016 at one token 10.0 us
+  // against 10.3 with start values, M = 16 11.0 against 11.3); a correction per 32 k for more than four groups in sixteen
+  // waves, which have no registers left for start values either (groups of 64: 11008 x 4096 at M = 16 10.4 against 11.0, 6528 x
+  // 36352 at one token 29.2 against 30.1); start values for the rest.
+  constexpr bool kRowSums = MT == 1 && GW <= 2 && D <= 4;
+  constexpr bool kCorrect = MT == 1 && GW > 4;
+  constexpr bool kStart = !kRowSums && !kCorrect;
   unsigned sz_off[SZR];
 #pragma unroll
   for (int r = 0; r < SZR; ++r) {
-    const int f = 64 * r + lane, i = f / (16 * GP), gq = (f >> 4) % GP;
-    const bool ok = i < NB && gq < GW && kt0 + gq / GPT < wg_end;
+    const int f = 64 * r + lane, i = f / (16 * GW), gq = (f >> 4) % GW;
+    const bool ok = i < NB && kt0 + gq / GPT < wg_end;
     sz_off[r] = ok ? (unsigned)i * sz_stride + (unsigned)gq * 64u + (unsigned)c * 4u : 0x80000000u;
   }
 
@@ -140,7 +139,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
       szraw[r] = __builtin_amdgcn_raw_buffer_load_b32(rs_sz, sz_off[r] + (unsigned)(batch * NB) * sz_stride, 0, 0);
   };
 
-  uint32_t m_lo = O::kMaskLo, m_hi = O::kMaskHi, c_lo = O::kMagicLo, c_hi = O::kMagicHi;
+  uint32_t m_lo = kStart ? O::kMask16 : O::kMaskLo, m_hi = O::kMaskHi, c_lo = kStart ? O::kMagic16 : O::kMagicLo, c_hi = O::kMagicHi;
   KSQ_PIN_SGPR(m_lo);
   KSQ_PIN_VGPR(c_lo);
   KSQ_PIN_VGPR(c_hi);
@@ -191,12 +190,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
   }
 
   // Bias and zero point: the nibbles enter the matrix instruction as bias + u, so every (column, group) owes
-  // -sum_k a_k (bias_k + z): added to a column tile's accumulators as a product over the groups (GroupCorrection), whose
-  // row operand is made here.  One row tile and at most two groups per wave: the two sums over the activations,
-  // sum_k a_k and -sum_k a_k bias_k, stay in registers in accumulator layout instead, and every group starts its
-  // accumulator from them -- with so few groups the product is mostly zeros (Llama-2-7B qkv at one token 7.4 us against
-  // 7.6, gate_up at M = 16 11.7 against 11.9; with four, Llama-3-70B gate_up at M = 16, the product 45.5 -> 42.6 against
-  // a correction instruction per 32 k, and with two row tiles, M = 27, 69.5 -> 63.7).
+  // -sum_k a_k (bias_k + z).  kRowSums: the two sums over the activations, sum_k a_k and -sum_k a_k bias_k, in accumulator layout.
+  // kStart: four registers a row tile with the rows' sums, one operand of the instruction that makes the start value.
   f32x4 asum[kRowSums ? TPW : 1][GPT], abias[kRowSums ? TPW : 1][GPT];
   if constexpr (kRowSums) {
     const uint32_t ones = O::kOnes;
@@ -214,29 +209,23 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
         }
       }
   }
-  // row sums of the wave's groups, lane 16 j + c = row c, group 4 q + j (or j % GP: see `sub` below)
-  float rsum[kRowSums ? 1 : MT][CG][kTerms];
-  if constexpr (!kRowSums) {
+  using Start = GroupStart<T>;
+  static_assert(!kStart || GW <= Start::kMaxGroups, "row sums of one wave");
+  const uint32_t start_base = Start::column_base(j);
+  u32x4 start_rows[MT];
+  if constexpr (kStart) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt) {
+      start_rows[mt] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int q = 0; q < CG; ++q)
+      for (int g = 0; g < GW; ++g) {
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int term = 0; term < kTerms; ++term) {
-        float v = 0.f;
-#pragma unroll
-        for (int g4 = 0; g4 < (GP < 4 ? GP : 4); ++g4) {
-          const int g = 4 * q + g4;
-          if (g >= GW) continue;
-          f32x4 d4 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int dd = 0; dd < DPG; ++dd)
-            d4 = Correction::accumulate(term, af[mt][g / GPT][(g % GPT) * DPG + dd], d4);
-          v = (GP < 4 ? j % GP : j) == g4 ? d4[0] : v;
-        }
-        rsum[mt][q][term] = v;
+        for (int dd = 0; dd < DPG; ++dd) sum = Start::sum(af[mt][g / GPT][(g % GPT) * DPG + dd], sum);
+        Start::fill(start_rows[mt], g, sum[0], j);
         __builtin_amdgcn_sched_barrier(0);  // all chains at once would not fit the registers beside the ring
       }
+    }
   }
 
   uint16_t* out = static_cast<uint16_t*>(p.out);
@@ -250,53 +239,55 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)
       for (int t = 0; t < TPW; ++t)
 #pragma unroll
         for (int gi = 0; gi < GPT; ++gi) {
-          const int f16 = i * GP + t * GPT + gi;  // flat word index / 16
+          const int f16 = (i * TPW + t) * GPT + gi;  // flat word index / 16
           szq[i * TPW + t][gi] =
               (uint32_t)__builtin_amdgcn_ds_bpermute(sz_lane + 64 * (f16 & 3), (int)szraw[f16 >> 2]);
         }
-    uint32_t szcol[kRowSums ? 1 : SZR];  // the words as loaded: the correction's column operands come from them
-#pragma unroll
-    for (int r = 0; r < (kRowSums ? 0 : SZR); ++r) szcol[r] = szraw[r];
     __builtin_amdgcn_sched_barrier(0);
     fetch_sz(b + 1);
     __builtin_amdgcn_sched_barrier(0);
-    f32x4 accb[NB][MT];
+    // The start values of group q of the batch (column tile, k tile, group of the k tile: all constants in the unrolled loops).
+    // A group's are made behind the matrix instructions of the one before: they need no weight, and the scaling waits there
+    // (4096 x 22016 at M = 32 14.3 -> 14.1 us).
+    auto start = [&](int q, f32x4 (&P)[MT]) __attribute__((always_inline)) {
+      const uint32_t szw = szq[q / GPT][q % GPT];
+      const int g = q % GW;
+      if constexpr (kRowSums) {
+        const float zf = (float)((szw >> 16) & 15u);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) P[0][e] = __builtin_fmaf(-zf, asum[g / GPT][g % GPT][e], abias[g / GPT][g % GPT][e]);
+      } else if constexpr (kCorrect) {
+        P[0] = f32x4{0.f, 0.f, 0.f, 0.f};
+      } else {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) P[mt] = Start::apply(start_rows[mt], start_base, g, szw, j);
+      }
+    };
+    f32x4 accb[NB][MT], next[MT];
+    start(0, next);
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        accb[i][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int q = 0; q < (kRowSums ? 0 : CG); ++q)
-#pragma unroll
-          for (int term = 0; term < kTerms; ++term) {
-            // an instruction that holds the words of several column tiles: the rows of the other tiles' groups are zero
-            const int r = GP >= 4 ? i * CG + q : i * GP / 4, sub = GP >= 4 ? 0 : i % (4 / GP);
-            const float rows = GP >= 4 || j / GP == sub ? rsum[mt][q][term] : 0.f;
-            accb[i][mt] = Correction::apply(rows, Correction::columns(term, szcol[r]), accb[i][mt]);
-          }
-      }
+      for (int mt = 0; mt < MT; ++mt) accb[i][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int t = 0; t < TPW; ++t) {
         const int slot = i * TPW + t;
 #pragma unroll
         for (int gi = 0; gi < GPT; ++gi) {
           const float s = O::scale_to_float(szq[slot][gi]);
+          const uint32_t z = (szq[slot][gi] >> 16) & 15u, zc = z | (z << 16);
           f32x4 P[MT];
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) P[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-          if constexpr (kRowSums) {
-            const float zf = (float)((szq[slot][gi] >> 16) & 15u);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) P[0][e] = __builtin_fmaf(-zf, asum[t][gi][e], abias[t][gi][e]);
-          }
+          for (int mt = 0; mt < MT; ++mt) P[mt] = next[mt];
 #pragma unroll
           for (int dd = 0; dd < DPG; ++dd) {
             const int d = gi * DPG + dd;
-            const u32x4 bw = kUniform ? O::unpack_uniform(wq[slot][d], m_lo, c_lo) : O::unpack(wq[slot][d], m_lo, m_hi, c_lo, c_hi);
+            const u32x4 bw = kStart ? O::unpack16(wq[slot][d], m_lo, c_lo) : O::unpack(wq[slot][d], m_lo, m_hi, c_lo, c_hi);
+            if constexpr (kCorrect) P[0] = O::mfma(af[0][t][d], O::correction(zc), P[0]);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) P[mt] = O::mfma(af[mt][t][d], bw, P[mt]);
           }
+          if (slot * GPT + gi + 1 < D * GPT) start(slot * GPT + gi + 1, next);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
 #pragma unroll

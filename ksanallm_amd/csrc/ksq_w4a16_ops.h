@@ -30,17 +30,16 @@ struct Ops<_Float16> {
   }
   static constexpr uint32_t kMaskLo = 0x000F000Fu, kMaskHi = 0x00F000F0u;
   static constexpr uint32_t kMagicLo = 0x64006400u, kMagicHi = 0x54005400u;
-  // the same word with every nibble in the 1024 + u form (two more shifts): one bias for all elements, so that
-  // sum a * (bias + z) factors into (bias + z) * sum a
-  static __device__ inline u32x4 unpack_uniform(uint32_t x, uint32_t m_lo, uint32_t c_lo) {
+  // the same word with every nibble as 16 + u (three more instructions): sums of biased products lose fewer low bits
+  static __device__ inline u32x4 unpack16(uint32_t x, uint32_t mask, uint32_t magic) {
     u32x4 v;
-    v[0] = (x & m_lo) | c_lo;
-    v[1] = ((x >> 4) & m_lo) | c_lo;
-    v[2] = ((x >> 8) & m_lo) | c_lo;
-    v[3] = ((x >> 12) & m_lo) | c_lo;
+    v[0] = ((x << 6) & mask) | magic;
+    v[1] = ((x << 2) & mask) | magic;
+    v[2] = ((x >> 2) & mask) | magic;
+    v[3] = ((x >> 6) & mask) | magic;
     return v;
   }
-  static constexpr float kBias = 1024.f;
+  static constexpr uint32_t kMask16 = 0x03C003C0u, kMagic16 = 0x4C004C00u;
   static constexpr uint32_t kOnes = 0x3C003C00u;
   // -(bias + z) per element for the correction MFMA; zc = z replicated into both halves
   static __device__ inline u32x4 correction(uint32_t zc) {
@@ -70,10 +69,16 @@ struct Ops<__bf16> {
   }
   static constexpr uint32_t kMaskLo = 0x000F000Fu, kMaskHi = 0x000F000Fu;
   static constexpr uint32_t kMagicLo = 0x43004300u, kMagicHi = 0x43004300u;
-  static __device__ inline u32x4 unpack_uniform(uint32_t x, uint32_t m_lo, uint32_t c_lo) {
-    return unpack(x, m_lo, m_lo, c_lo, c_lo);
+  // 16 + u, the nibble in the upper bits of the mantissa (one more shift): sums of biased products lose fewer low bits
+  static __device__ inline u32x4 unpack16(uint32_t x, uint32_t mask, uint32_t magic) {
+    u32x4 v;
+    v[0] = ((x << 3) & mask) | magic;
+    v[1] = ((x >> 1) & mask) | magic;
+    v[2] = ((x >> 5) & mask) | magic;
+    v[3] = ((x >> 9) & mask) | magic;
+    return v;
   }
-  static constexpr float kBias = 128.f;
+  static constexpr uint32_t kMask16 = 0x00780078u, kMagic16 = 0x41804180u;
   static constexpr uint32_t kOnes = 0x3F803F80u;
   static __device__ inline u32x4 correction(uint32_t zc) {
     const uint32_t v = 0xC300C300u | zc;
@@ -87,32 +92,56 @@ struct Ops<__bf16> {
   static __device__ inline uint16_t to_bits(float v) { return __builtin_bit_cast(uint16_t, (__bf16)v); }
 };
 
-// Bias and zero point of biased nibbles, for a whole (column tile, row tile) at once.  The matrix instructions see
-// bias_k + u instead of u - z, so the sum over a group owes -sum_k a_k (bias_k + z), and scaled by the group's s
-//   -s z sum_k a_k - s sum_k a_k bias_k = sum over groups of (row factor) x (column factor):
-// a matrix product whose k index is the group.  v_mfma_f32_16x16x4_f32 adds four groups of it to an accumulator in one
-// fp32 instruction.  Its operands are one register each: lane 16 j + c holds the row sums of row c over group j (made
-// once per wave), and the column factors of column c in group j (`columns`), which is how the scale/zero
-// words are loaded.  One or two such instructions per 512 k instead of a second 16x16x32 one for every 32 k.
-// UNIFORM: one bias for all k (bf16, and fp16 through unpack_uniform), so that one term does: -s (bias + z) sum_k a_k.
-template <typename T, bool UNIFORM>
-struct GroupCorrection {
-  static_assert(UNIFORM || __is_same(T, _Float16), "bf16 nibbles have one bias");
-  static constexpr int kTerms = UNIFORM ? 1 : 2;
-  // sum_k a_k for term 0, -sum_k a_k bias_k for term 1, of the row whose fragment is `frag`: D[m][n] with the
-  // constant as the first operand and the activations as the second has the row in its column index, the same in
-  // every register
-  static __device__ inline f32x4 accumulate(int term, u32x4 frag, f32x4 acc) {
-    if (term == 0) return Ops<T>::mfma(u32x4{Ops<T>::kOnes, Ops<T>::kOnes, Ops<T>::kOnes, Ops<T>::kOnes}, frag, acc);
-    return Ops<T>::mfma(Ops<T>::correction(0u), frag, acc);  // the negative biases
+// Bias and zero point of a group of nibbles unpacked by unpack16: the matrix instructions see 16 + u instead of u - z, so a
+// group's sum owes -(16 + z) S, S = sum_k a_k.  That is the group's start value, before its scale: it does not overflow where the
+// result does not, and a scale that is not finite stays in its own column.  One more of the matrix instructions that the sum itself
+// is made of gives it for a (column tile, row tile), from exact products: S as three 16-bit pieces against -(16 + z).
+//   rows    four registers, lane 16 j + c = row c; register q: group 2 q for j = 0, 1, group 2 q + 1 for j = 2, 3, the pieces
+//           (1, 2) for even, (3, 0) for odd j.  bf16: the upper, middle and lower eight bits of S.  fp16: S = 2^8 p1 + 2^-2 p2 +
+//           2^-12 p3, exact because S is at most 2^23 and a multiple of 2^-24, like every fp16 activation
+//   column  four registers, lane 16 j + c = column c: -(16 + z) times the piece's power of two in the group's register and
+//           lanes, zero elsewhere (a row whose sum is not finite is lost in every group)
+// (The same from v_mfma_f32_16x16x16_bf16, half the k, gave wrong values in the upper two registers of some accumulators, from run
+// to run: a 16x16x32 sum must not start from it.)
+template <typename T>
+struct GroupStart {
+  static constexpr bool kF16 = __is_same(T, _Float16);
+  static constexpr int kMaxGroups = 8;
+  // S of the row whose fragment is `frag`: D[m][n] with ones as the first operand and the activations as the second has the row
+  // in its column index, the same in every register
+  static __device__ inline f32x4 sum(u32x4 frag, f32x4 acc) {
+    return Ops<T>::mfma(u32x4{Ops<T>::kOnes, Ops<T>::kOnes, Ops<T>::kOnes, Ops<T>::kOnes}, frag, acc);
   }
-  static __device__ inline float columns(int term, uint32_t szw) {
-    const float s = Ops<T>::scale_to_float(szw), z = (float)((szw >> 16) & 15u);
-    if constexpr (kTerms == 1) return -s * (Ops<T>::kBias + z);
-    return term == 0 ? -s * z : s;
+  // group g's sum into its register and lanes
+  static __device__ inline void fill(u32x4& rows, int g, float s, int j) {
+    uint32_t p12, p3;
+    if constexpr (kF16) {
+      const _Float16 p1 = (_Float16)(s * 0x1p-8f);
+      const float r = s - (float)p1 * 0x1p8f;
+      const _Float16 p2 = (_Float16)(r * 0x1p2f);
+      const _Float16 l = (_Float16)((r - (float)p2 * 0x1p-2f) * 0x1p12f);
+      p12 = (uint32_t)__builtin_bit_cast(uint16_t, p1) | (uint32_t)__builtin_bit_cast(uint16_t, p2) << 16;
+      p3 = __builtin_bit_cast(uint16_t, l);
+    } else {
+      const uint32_t p1 = __builtin_bit_cast(uint32_t, s) & 0xFFFF0000u;
+      const float r = s - __builtin_bit_cast(float, p1);
+      const uint32_t p2 = __builtin_bit_cast(uint32_t, r) & 0xFFFF0000u;
+      p12 = p1 >> 16 | p2;
+      p3 = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, p2)) >> 16;
+    }
+    const uint32_t mine = (j & 1) ? p3 : p12;
+    rows[g >> 1] = (j >> 1) == (g & 1) ? mine : rows[g >> 1];
   }
-  static __device__ inline f32x4 apply(float row_sums, float cols, f32x4 acc) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(row_sums, cols, acc, 0, 0, 0);
+  // -16 times the pieces' powers of two, for this lane
+  static __device__ inline uint32_t column_base(int j) {
+    if constexpr (kF16) return (j & 1) ? 0x9C009C00u : 0xC400EC00u;
+    return 0xC180C180u;
+  }
+  static __device__ inline f32x4 apply(u32x4 rows, uint32_t base, int g, uint32_t szw, int j) {
+    const uint32_t c = ((szw >> 16) & 15u) * (kF16 ? 0x00400040u : 0x00080008u) + base;
+    u32x4 column = {0u, 0u, 0u, 0u};
+    column[g >> 1] = (j >> 1) == (g & 1) ? c : 0u;
+    return Ops<T>::mfma(rows, column, f32x4{0.f, 0.f, 0.f, 0.f});
   }
 };
 

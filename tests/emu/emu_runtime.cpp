@@ -543,7 +543,6 @@ void mfma_collective(WaveState* w, int slot, int kind) {
     case kMfmaF16:
     case kMfmaBf16:
     case kMfmaFp8x32: per_lane = 8; break;
-    case kMfmaF32: per_lane = 1; break;
     default: per_lane = 32; break;
   }
   static thread_local float A[16][128], B[16][128];
@@ -561,9 +560,6 @@ void mfma_collective(WaveState* w, int slot, int kind) {
         std::memcpy(&bh, &bb, 2);
         av = (float)ah;
         bv = (float)bh;
-      } else if (kind == kMfmaF32) {
-        std::memcpy(&av, a, 4);
-        std::memcpy(&bv, b, 4);
       } else if (kind == kMfmaBf16) {
         const uint32_t ab = (a[e >> 1] >> (16 * (e & 1))) << 16, bb = (b[e >> 1] >> (16 * (e & 1))) << 16;
         std::memcpy(&av, &ab, 4);

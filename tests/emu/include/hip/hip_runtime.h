@@ -148,7 +148,7 @@ extern float e4m3_table[256];
 uint8_t f32_to_e4m3(float v);
 
 void mfma_collective(WaveState* w, int slot, int kind);  // kinds below
-constexpr int kMfmaF16 = 0, kMfmaBf16 = 1, kMfmaFp8x32 = 2, kMfmaFp8x128 = 3, kMfmaF32 = 4;
+constexpr int kMfmaF16 = 0, kMfmaBf16 = 1, kMfmaFp8x32 = 2, kMfmaFp8x128 = 3;
 
 template <int WORDS>
 inline f32x4_t mfma(const void* a, const void* b, f32x4_t c, int kind, int site) {
@@ -270,10 +270,6 @@ inline emu::f32x4_t __builtin_amdgcn_mfma_f32_16x16x32_f16(emu_half8 a, emu_half
 inline emu::f32x4_t __builtin_amdgcn_mfma_f32_16x16x32_bf16(emu_bf16x8 a, emu_bf16x8 b, emu::f32x4_t c, int, int, int,
                                                            int site = __builtin_LINE()) {
   return emu::mfma<4>(&a, &b, c, emu::kMfmaBf16, site);
-}
-inline emu::f32x4_t __builtin_amdgcn_mfma_f32_16x16x4f32(float a, float b, emu::f32x4_t c, int, int, int,
-                                                         int site = __builtin_LINE()) {
-  return emu::mfma<1>(&a, &b, c, emu::kMfmaF32, site);
 }
 inline emu::f32x4_t __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(long a, long b, emu::f32x4_t c, int, int, int,
                                                               int site = __builtin_LINE()) {

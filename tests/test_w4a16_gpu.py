@@ -126,6 +126,79 @@ def test_k_stationary_split_sums(gpu, dtype, g, M, ksplit, per_wg):
     assert np.array_equal(got1, got2)
 
 
+# kernel forms of a decode call by how they remove bias and zero point: (rows, K, group size, overrides)
+_DECODE_FORMS = {
+    "row_sums": (16, 1024, 128, {}),                                                # k-stationary, up to two groups a wave
+    "start_1": (5, 4096, 64, {"KSQ_W4_KPHASE": 0}),                                 # k-stationary, one row tile, four groups
+    "correction": (1, 8192, 64, {"KSQ_W4_KPHASE": 0, "KSQ_W4_KSTAT_TPW_MAX": 4}),    # ... eight
+    "start_1_split": (16, 8192, 128, {"KSQ_W4_KSPLIT": 2, "KSQ_W4_KSTAT_NT_PER_WG": 4}),  # two groups, four column tiles a batch
+    "start_2": (27, 1024, 128, {"KSQ_W4_ASTREAM": 0, "KSQ_W4_KSTAT_NT_PER_WG": 4}),  # two row tiles, two groups, batches of two
+    "start_2_eight": (27, 4096, 64, {"KSQ_W4_ASTREAM": 0}),                        # ... eight
+    "start_4": (50, 2048, 128, {"KSQ_W4_ASTREAM": 0, "KSQ_W4_KSTAT_NT_PER_WG": 2}),
+    "phases": (3, 2176, 128, {"KSQ_W4_KPHASE": 1}),
+    "astream": (40, 1024, 128, {"KSQ_W4_ASTREAM": 1, "KSQ_W4_ASTREAM_LDS": 0}),
+    "astream_lds": (20, 1024, 64, {"KSQ_W4_ASTREAM": 1, "KSQ_W4_ASTREAM_LDS": 1}),
+    "stream": (9, 1024, 128, {"KSQ_W4_KSTAT": 0}),
+}
+
+
+@pytest.mark.parametrize("form", _DECODE_FORMS)
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_a_scale_that_is_not_finite_stays_in_its_column(gpu, form, dtype):
+    """An infinite and a NaN group scale: every other column is what it is without them, bit for bit."""
+    M, K, g, env = _DECODE_FORMS[form]
+    N, hit = 336, (5, 40, 200)
+    rng = np.random.default_rng(1460 + M)
+    sv = np.abs(rng.standard_normal((K // g, N))).astype(np.float32) * 0.02 + 1e-3
+    with _env(**env):
+        want = W4Device(W4Case(1461, M, K, N, g=g, kind="awq", dtype=dtype, scales=sv), gpu).gemm_f32()
+        sv = sv.copy()
+        sv[0, hit[0]], sv[-1, hit[1]], sv[K // g // 2, hit[2]] = np.inf, np.nan, -np.inf
+        got = W4Device(W4Case(1461, M, K, N, g=g, kind="awq", dtype=dtype, scales=sv), gpu).gemm_f32()
+    others = np.setdiff1d(np.arange(N), hit)
+    assert np.all(np.isfinite(want)) and np.array_equal(got[:, others], want[:, others]), \
+        np.unique(np.nonzero(~np.isfinite(got))[1])
+    assert not np.any(np.isfinite(got[:, hit]))
+
+
+@pytest.mark.parametrize("form", _DECODE_FORMS)
+def test_scales_near_the_end_of_the_bf16_range(gpu, form):
+    """Scales of 1e36 and activations with a sum of 3 over a group: what is owed for bias and zero point, scaled, is
+    (128 + 8) 1e36 3 with bf16's usual bias, not a finite float, while no result is beyond 2.3e38."""
+    M, K, g, env = _DECODE_FORMS[form]
+    rng = np.random.default_rng(1470 + M)
+    sv = (1e36 * (1 + 0.1 * rng.random((K // g, 336)))).astype(np.float32)
+    act = (3.0 / g * (1 + 0.3 * rng.standard_normal((M, K)))).astype(np.float32)
+    case = W4Case(1471, M, K, 336, g=g, kind="gptq", dtype="bf16", scales=sv, act=act)
+    with _env(**env):
+        got = W4Device(case, gpu).gemm_f32()
+    assert np.all(np.isfinite(got))
+    orc.assert_parity(got * np.float32(1e-36), case.oracle() * np.float32(1e-36), f"scales of 1e36, {form}")
+
+
+@pytest.mark.parametrize("form", ["start_1", "start_2", "start_2_eight", "start_4"])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_decode_sums_round_to_the_exact_result(gpu, form, dtype):
+    """How many outputs are not the correctly rounded exact result.  With activations of mean 2 a group's biased sum is some
+    d = 2 g (16 + 7.5) against a result around sqrt(5 K) 6.5 s: five fp32 roundings of up to half an ulp of d a group, taken as
+    independent, are an error of e = 2^-24 d s sqrt(5 K / g / 3) (rms), and an output is off with probability e / ulp.  Twice that
+    is allowed; sums that carry a bias of 1024 (fp16) or 128 (bf16) through all groups of a wave have six times as many."""
+    M, K, g, env = _DECODE_FORMS[form]
+    M, N, s = max(M, 16) if form == "start_1" else M, 1040 if M < 20 else 528, 0.02
+    rng = np.random.default_rng(1480 + M)
+    act = (2 + rng.standard_normal((M, K))).astype(np.float32)
+    sv = (s * np.exp(0.25 * rng.standard_normal((K // g, N)))).astype(np.float32)
+    case = W4Case(1481, M, K, N, g=g, kind="awq", dtype=dtype, scales=sv, act=act)
+    with _env(**env):
+        got = bits_of(W4Device(case, gpu).gemm())
+    w = (case.u.astype(np.float64) - np.repeat(case.z, g, 0)) * np.repeat(orc.from_bits(case.scales, ORC_DT[dtype]), g, 0)
+    exact = orc.from_bits(case.act, ORC_DT[dtype]).astype(np.float64) @ w
+    off = np.mean(got != orc.to_bits(exact.astype(np.float32), ORC_DT[dtype]))
+    result, bits = np.sqrt(5.0 * K) * 6.5 * s, {"f16": 10, "bf16": 7}[dtype]
+    e = 2.0 ** -24 * 2 * g * (16 + 7.5) * s * np.sqrt(5 * K / g / 3)
+    assert off <= 2 * e / (result * 2.0 ** -bits), (off, e / (result * 2.0 ** -bits))
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("kind,g", [("gptq", 128), ("gptq", 64), ("awq", 64)])
 def test_group_sizes_and_kinds(gpu, dtype, kind, g):
