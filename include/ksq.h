@@ -297,10 +297,11 @@ int ksq_fp8_gemm_ex(int out_dtype, void* out, const void* act_q, const float* ac
  *   out[m,n] = T( (sum_k a_q[m,k] * w[n,k]) * w_scale[n or 0] * scale[m] ),
  * i.e. ksq_fp8_quantize(KSQ_FP8_PER_TOKEN_DYNAMIC) followed by ksq_fp8_gemm_ex, which is what it runs for m > 1: one
  * call for the reference's Fp8E4m3Quantize + Fp8QuantizedMatMul pair (KS/kernels/nvidia/kernel_wrapper.cpp:1015-1041,
- * KS/layers/nvidia/fp8_matmul_layer.cpp:56-63).  A single token (k a multiple of 128, at most 8192) is one launch:
- * every workgroup takes the row maximum and quantises the activations itself, with the same arithmetic, so the
- * quantised bytes are those of ksq_fp8_quantize.  (Measured, that form only ties with the two launches at one row and
- * loses from two rows on, since every workgroup repeats the quantisation; it can do up to eight rows.)  The workspace
+ * KS/layers/nvidia/fp8_matmul_layer.cpp:56-63).  A single token (k a multiple of 128, at most 8192) can be one
+ * launch, and is where that is the faster form or no workspace is given: every workgroup takes the row maximum and
+ * quantises the activations itself, with the same arithmetic, so the quantised bytes are those of ksq_fp8_quantize.
+ * (Measured, that form wins a few per cent on some shapes at one row, loses as much on others, and loses from two rows
+ * on, since every workgroup repeats the quantisation; it can do up to eight rows.)  The workspace
  * (ksq_fp8_gemm_dynamic_workspace_bytes, 256-byte aligned) holds the quantised activations and scales of the two-launch
  * route and the split-K partial sums; without one only the single-launch case works, anything else fails with
  * KSQ_ERR_WORKSPACE. */

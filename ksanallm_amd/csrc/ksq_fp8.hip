@@ -813,7 +813,8 @@ int ksq_fp8_gemm_dynamic(int dtype, void* out, const void* act, const void* w_q,
   const size_t fused_rows = sw ? (atoi(sw) == 0 ? 0 : 8) : 1;
   const size_t cus16 = 16 * (size_t)di->cus;
   const bool worth = k >= 4096 && n > cus16 && (k < 8192 || n > 2 * cus16) && (n <= 3 * cus16 || k % 4096 == 0);
-  if (m <= fused_rows && (sw || worth) && dtype != KSQ_F32 && k % 128 == 0 && m * k * 2 < 0x7FFFFF00ull) {
+  const bool alone = workspace_bytes < front;  // no place for quantised activations: the one launch is all there is
+  if (m <= fused_rows && (sw || worth || alone) && dtype != KSQ_F32 && k % 128 == 0 && m * k * 2 < 0x7FFFFF00ull) {
     if (gemm_ws && !counter_slot_available(s)) gemm_ws = nullptr, gemm_ws_bytes = 0;
     const Fp8KstatPlan kp = fp8_kstat_plan(m, n, k, di->cus, gemm_ws_bytes, true);
     if (kp.ok && kp.nb <= 2 && kp.tpw <= 4 && (kp.ksplit == 1 || sw)) {

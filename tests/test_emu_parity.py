@@ -92,6 +92,7 @@ test_gemm_large_m_small_integers_exact = f8.test_gemm_large_m_small_integers_exa
 test_gemm_small_integers_exact = f8.test_gemm_small_integers_exact
 test_convert_weight_per_channel = f8.test_convert_weight_per_channel
 test_merge_qkv_scales = f8.test_merge_qkv_scales
+test_gemm_dynamic_one_token_needs_no_workspace = f8.test_gemm_dynamic_one_token_needs_no_workspace
 test_gemm_dynamic_quantiser_is_the_quantise_kernels = f8.test_gemm_dynamic_quantiser_is_the_quantise_kernels
 test_gemm_dynamic_epilogues_and_errors = f8.test_gemm_dynamic_epilogues_and_errors
 

@@ -652,6 +652,21 @@ def test_gemm_dynamic_quantises_inside(gpu, dtype, M, K, N):
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("K,N", [(128, 64), (1024, 272), (2048, 4096), (4096, 4096), (5120, 528), (8192, 1040)])
+def test_gemm_dynamic_one_token_needs_no_workspace(gpu, dtype, K, N):
+    """One token, K a multiple of 128 up to 8192, no workspace: one launch, also where the library prefers two."""
+    rng = np.random.default_rng(465 + K)
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    ws = orc.fp8_compute_scale(w, orc.F32, N, K)
+    wq = orc.fp8_quantize(w, orc.F32, ws, N, K)
+    x = orc.to_bits(rng.standard_normal((1, K)).astype(np.float32), ORC_DT[dtype])
+    got = _run_dynamic(gpu, x, wq, ws, dtype, use_workspace=False)
+    xs = orc.fp8_compute_scale(x, ORC_DT[dtype], 1, K)
+    xq = orc.fp8_quantize(x, ORC_DT[dtype], xs, 1, K)
+    orc.assert_parity(got.float().cpu().numpy(), orc.fp8_gemm(xq, xs, wq, ws), f"fp8 dynamic, no workspace K={K} N={N}")
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("M", [1, 4, 8])
 def test_gemm_dynamic_quantiser_is_the_quantise_kernels(gpu, dtype, M):
     """An identity weight (e4m3 1.0 on the diagonal, scale 1) turns the GEMM into out[m, k] = T(float(q[m, k]) * scale[m]):
