@@ -34,6 +34,9 @@ HIPCC_FLAGS = [
 # the compiler ever stops inlining one of those lambdas the captures move to memory (seen once: 1136 bytes per lane and
 # a tenth of the speed, with every test still passing).  Real register spills of the fallback kernels stay below this.
 MAX_SCRATCH_BYTES = 512
+# The tile kernel's steps have no memory instruction to spare: its forms spill at most 20 registers (two k groups, 128 x 64 a
+# wave; counted in the planner's estimates).  31 in one form that the estimates did not know of cost 40 %.
+MAX_SCRATCH_BYTES_OF = {"w4a16_prefill_kernel": 88}
 
 
 def check_scratch(src, remarks):
@@ -45,9 +48,10 @@ def check_scratch(src, remarks):
             name = text.split(":", 1)[1].split("[")[0].strip()
         elif text.startswith("ScratchSize"):
             size = int(text.split(":", 1)[1].split("[")[0].strip())
-            if size > MAX_SCRATCH_BYTES:
-                raise RuntimeError(f"{src}: kernel {name} uses {size} bytes of scratch memory per lane "
-                                   f"(limit {MAX_SCRATCH_BYTES}): a lambda of the kernel is probably no longer inlined")
+            limit = next((v for k, v in MAX_SCRATCH_BYTES_OF.items() if k in (name or "")), MAX_SCRATCH_BYTES)
+            if size > limit:
+                raise RuntimeError(f"{src}: kernel {name} uses {size} bytes of scratch memory per lane (limit {limit}): "
+                                   "spilled registers, or a lambda of the kernel that is no longer inlined")
 
 
 def hipcc():

@@ -57,7 +57,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
   using O = Ops<_Float16>;  // the matrix cores run in fp16 for both element types
   using DQ = Dequant<T>;
   constexpr bool kBF16 = sizeof(T) == 2 && !__is_same(T, _Float16);
-  constexpr int kStage = RT * 4 * 64;  // 16-byte elements per activation stage (16 RT rows x 128 k): 32 KiB with eight
+  // 16-byte elements per activation stage (16 RT rows x 128 k): 32 KiB with eight.  Where the waves do not divide the blocks
+  // (eight waves with five or seven row tiles) a stage has room for kFPW blocks from every wave, and the last ones' go unread:
+  // a branch around those loads split every step for the compiler, which then spilled 31 registers with groups of 64 (us, with
+  // the branch / without: M = 1774, 4096 x 16320 fp16 271 / 192, bf16 290 / 201; groups of 128, not spilled, 189 / 186; five
+  // row tiles, M = 144, 4096 x 32976 50.7 / 51.9).
+  constexpr int kStage = kFPW * NW * 64;
   constexpr int kEpiStride = 68;        // floats per row of the epilogue transpose (2-way conflicts at worst)
   // two activation stages as two separate objects: loads into one are then known not to alias reads of the other
   __shared__ u32x4 lds_a0[kStage];
@@ -138,7 +143,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
 #pragma unroll
     for (int x = 0; x < kPart; ++x) {
       const int i = kPart * q + x;
-      if (i < kFPW && (kFPW * NW == 4 * RT || kFPW * wave + i < 4 * RT))
+      if (i < kFPW)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (lds_ptr)(buf + (kFPW * wave + i) * 64), 16, a_off[i], kt * 256, 0, 0);
     }
   };

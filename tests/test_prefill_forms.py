@@ -47,3 +47,18 @@ def test_no_other_form_is_compiled():
     got = {(t, int(gpt), *(int(v) for v in form)) for t, gpt, *form in found}
     want = {(t, gpt, *form) for t in ("DF16_", "DF16b") for gpt in (1, 2) for form in FORMS}
     assert got == want, (sorted(got - want), sorted(want - got))
+
+
+def test_the_build_refuses_spilling_forms():
+    """What the compiler says of a form that spills 31 registers (124 bytes a lane) stops the build; 20 (84) do not."""
+    import pytest
+
+    from ksanallm_amd import build
+
+    def remarks(size):
+        return [f"f.h:1:1: remark: Function Name: _ZN3ksq20w4a16_prefill_kernelIDF16bLi2EEEv [-Rpass-analysis=x]",
+                f"f.h:1:1: remark:     ScratchSize [bytes/lane]: {size} [-Rpass-analysis=x]"]
+
+    build.check_scratch("f.hip", remarks(84))
+    with pytest.raises(RuntimeError, match="124 bytes"):
+        build.check_scratch("f.hip", remarks(124))
