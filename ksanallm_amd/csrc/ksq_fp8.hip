@@ -804,15 +804,15 @@ int ksq_fp8_gemm_dynamic(int dtype, void* out, const void* act, const void* w_q,
   // Every one of its workgroups repeats that work, so it only ties with the two launches at a single row without a
   // split of K (Qwen-72B qkv: 22.2 us against 3.0 + 19.3) and loses beyond (two rows 23.5 against 22.5, eight rows
   // 29.9 against 23.6; K = 29568, split four ways: 65.9 against 59.3): it serves m = 1, and up to eight rows on request.
-  // At one row it wins where a workgroup has something to hide the quantisation behind and a row is long enough for the
-  // other launch to matter (ratio two launches / one over K = 2176 .. 8192, N = 2048 .. 32768, both types):
-  //   K < 4096 0.85 .. 1.00 everywhere; one column tile per CU and fewer 0.85 .. 0.92; two 1.02 .. 1.11, but 0.88 at
-  //   K = N = 8192; three 0.99 .. 1.04; more 1.00 .. 1.06 where K is a multiple of 4096, so that every wave has the same
-  //   number of k tiles, and 0.97 .. 0.99 elsewhere.
+  // At one row (ratio two launches / one over K = 2048 .. 8192, N = 2048 .. 59136, bf16):
+  //   K < 4096 0.85 .. 1.01, one column tile per CU and fewer 0.87 .. 0.89: a workgroup has too little else to do;
+  //   two column tiles per CU 1.04 .. 1.10 for K = 4096 .. 7168, but 0.98 and 0.88 at 8192;
+  //   three and more 0.98 .. 1.02 at K = 4096, 0.99 .. 1.00 at 8192, 0.97 .. 0.99 at 5120, 6144 and 7168.  (The waves' equal
+  //   shares are not the reason: 6144 has them too.)  Where it is level, one launch.
   const char* sw = tuning_env("KSQ_FP8_FUSED_QUANT");  // tuning / test switch: 0 = never, 1 = up to eight rows
   const size_t fused_rows = sw ? (atoi(sw) == 0 ? 0 : 8) : 1;
   const size_t cus16 = 16 * (size_t)di->cus;
-  const bool worth = k >= 4096 && n > cus16 && (k < 8192 || n > 2 * cus16) && (n <= 3 * cus16 || k % 4096 == 0);
+  const bool worth = k >= 4096 && n > cus16 && (n <= 2 * cus16 ? k < 8192 : k % 4096 == 0);
   const bool alone = workspace_bytes < front;  // no place for quantised activations: the one launch is all there is
   if (m <= fused_rows && (sw || worth || alone) && dtype != KSQ_F32 && k % 128 == 0 && m * k * 2 < 0x7FFFFF00ull) {
     if (gemm_ws && !counter_slot_available(s)) gemm_ws = nullptr, gemm_ws_bytes = 0;
