@@ -145,10 +145,11 @@ __device__ inline ksq_f32x4 load_agent(const ksq_f32x4* p) {
 
 // Sum of V neighbouring 16-byte pieces over the splits, added in split order.  load(split, v) = piece v of that split's
 // partial tile.  The pieces of up to eight splits are requested together: one at a time, every split costs a whole trip
-// to the memory beyond the XCD's L2 (1.6 us each measured, against 0.2 for the ones after the first like this).  BATCH = 2 for
-// kernels that have no registers to spare.
+// to the memory beyond the XCD's L2 (1.6 us each measured, against 0.2 for the ones after the first like this).  BATCH = 8 or 2;
+// 2 for kernels that have no registers to spare.
 template <int V, int BATCH = 8, typename Load>
 __device__ inline void sum_splits(ksq_f32x4 (&sum)[V], int ksplit, Load load) {
+  static_assert(BATCH == 8 || BATCH == 2, "batches");
   int sp = 0;
 #pragma unroll
   for (int v = 0; v < V; ++v) sum[v] = ksq_f32x4{0.f, 0.f, 0.f, 0.f};
@@ -162,7 +163,7 @@ __device__ inline void sum_splits(ksq_f32x4 (&sum)[V], int ksplit, Load load) {
       _Pragma("unroll") for (int v = 0; v < V; ++v) sum[v] += part[q][v]; \
     sp += N;                                                    \
   } while (0)
-  if constexpr (BATCH >= 8) {
+  if constexpr (BATCH == 8) {
     while (sp + 8 <= ksplit) KSQ_SUM_BATCH(8);
     if (sp + 4 <= ksplit) KSQ_SUM_BATCH(4);
   }
@@ -216,7 +217,8 @@ __device__ inline bool splitk_arrive_last(unsigned* counter, int lane, int kspli
 // one or two batches of column tiles that one row tile leaves a workgroup, the arrivals of the first overlap the work of
 // the second and the late sum is the slower one (W4 o at M = 16 11.4 against 11.8 us, FP8 down 52 against 57).
 // Every wave of the workgroup makes the call; `load(sp, q)` = this lane's piece of tile q of split sp, `finish(q, sum)`
-// stores it.
+// stores it.  (Partial tiles of two splits requested together: with four, 16384 x 24576 at M = 24, four splits, 50.4 us against
+// 50.3, 28672 x 32768 at M = 27, seven, 116.1 and 116.1.)
 template <int NW, typename Load, typename Finish>
 __device__ inline void splitk_finish_workgroup(unsigned* counter, int wave, int lane, int ksplit, int tiles, Load load,
                                                Finish finish) {
@@ -232,13 +234,13 @@ __device__ inline void splitk_finish_workgroup(unsigned* counter, int wave, int 
   int q = wave;
   for (; q + NW < tiles; q += 2 * NW) {
     ksq_f32x4 sum[2];
-    sum_splits<2, 4>(sum, ksplit, [&](int sp, int v) { return load(sp, q + v * NW); });
+    sum_splits<2, 2>(sum, ksplit, [&](int sp, int v) { return load(sp, q + v * NW); });
     finish(q, sum[0]);
     finish(q + NW, sum[1]);
   }
   if (q < tiles) {
     ksq_f32x4 sum[1];
-    sum_splits<1, 4>(sum, ksplit, [&](int sp, int) { return load(sp, q); });
+    sum_splits<1, 2>(sum, ksplit, [&](int sp, int) { return load(sp, q); });
     finish(q, sum[0]);
   }
   if (wave == 0 && lane == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
