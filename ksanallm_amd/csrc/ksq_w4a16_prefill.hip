@@ -185,7 +185,10 @@ double estimate_eight_waves(int ct, int rt, size_t workgroups, int cus, size_t k
   const double us =
       ct == 3 ? 7.54 + (double)kt * ((double)full * (0.551 + 0.264 * rt) + (rem ? 0.395 + 0.124 * rt + 0.121 * rt * fill : 0.0))
               : 7.77 + (double)kt * ((double)full * (0.669 + 0.350 * rt) + (rem ? 0.671 + 0.143 * rt + 0.153 * rt * fill : 0.0));
-  // whole rounds (M = 4096 of the 7B shapes): the fit, made mostly of grids with a rest, is 3 to 5 % too high for them
+  // Grids of whole rounds: the fit, made mostly of grids with a rest, is some 4 % too high for them (no CU waits for the last
+  // round's tail).  Where that decides against the next form -- 49 of 3960 shapes, four waves in 45 of them -- eight waves in
+  // whole rounds were 2.5 % faster on average (48 measured): M = 4096, 4096 x 4096 107.9 against 113.0 us, M = 967, 1152 x 16336 36.6 against 38.9,
+  // M = 2019, 4864 x 6080 98.9 against 107.4; slower in eight, by 7 % at most (M = 3516, 1280 x 44816 375 against 350).
   return rem == 0 ? 0.96 * us : us;
 }
 
