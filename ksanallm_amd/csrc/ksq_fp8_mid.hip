@@ -281,14 +281,7 @@ constexpr MidForm kForms[] = {
 constexpr double kReduce = 1.89, kReduceMB = 0.29;
 constexpr size_t kMaxM = 2048;  // fitted up to here; the 256-row tiles win from about 1000 rows on anyway
 
-double mid_estimate(const MidForm& f, size_t m, size_t n, size_t k, size_t ks, size_t cus) {
-  const size_t mb = (m + 16 * f.mt - 1) / (16 * f.mt), nb = (n + 128 * f.wn - 1) / (128 * f.wn);
-  const size_t wgs = (mb * nb + 7) / 8 * 8 * ks, rounds = (wgs + cus - 1) / cus, stages = ((k + 127) / 128 + ks - 1) / ks;
-  const double busy = (double)wgs / (double)(cus * rounds);
-  double t = f.fixed + rounds * (f.round + stages * (f.stage + f.load * busy));
-  if (ks > 1) t += kReduce + kReduceMB * 1e-6 * ks * ((m + 15) / 16 * 16) * n * 4;
-  return t;
-}
+constexpr size_t kMaxSplit = 12;
 
 // The decode kernels at 17 .. 64 rows: a fixed part, the weights, the activations that every workgroup pulls (10 % rms)
 double kstat_estimate(size_t m, size_t n, size_t k) {
@@ -322,16 +315,28 @@ Fp8MidPlan fp8_mid_plan(size_t m, size_t n, size_t k, int cus_, size_t workspace
     else if (k % 128 == 0) limit = fp8_prefill_estimate(m, n, k, cus_);
     // else: the alternative is the streaming kernel, five to ten times as slow
   }
+  // This runs in every call of these sizes (0.9 us with every estimate made in full): a form and split whose stages alone take
+  // longer than the best so far goes no further.
+  size_t split_stages[kMaxSplit + 1];
+  for (size_t ks = 1; ks <= kMaxSplit; ++ks) split_stages[ks] = (stages + ks - 1) / ks;
   for (int f = 0; f < (int)(sizeof(kForms) / sizeof(kForms[0])); ++f) {
     if (form >= 0 && f != form) continue;
-    for (size_t ks = 1; ks <= 12 && (ks == 1 || ks * 4 <= stages || ks == splits); ++ks) {
+    const MidForm& fm = kForms[f];
+    const size_t mb = (m + 16 * fm.mt - 1) / (16 * fm.mt), nb = (n + 128 * fm.wn - 1) / (128 * fm.wn);
+    const size_t tiles = (mb * nb + 7) / 8 * 8;
+    for (size_t ks = 1; ks <= kMaxSplit && (ks == 1 || ks * 4 <= stages || ks == splits); ++ks) {
       if (splits && ks != splits) continue;
       const size_t need = ks > 1 ? ks * mtiles * ntiles * 1024 : 0;
       if (need > workspace_bytes || ks > stages) break;
-      const double t = mid_estimate(kForms[f], m, n, k, ks, cus);
+      const double reduce = ks > 1 ? kReduce + kReduceMB * 1e-6 * (double)(ks * mtiles * 16 * n * 4) : 0.0;
+      if (fm.fixed + fm.round + (double)split_stages[ks] * fm.stage + reduce >= limit) continue;
+      const size_t wgs = tiles * ks, rounds = (wgs + cus - 1) / cus;
+      const double busy = (double)wgs / (double)(cus * rounds);
+      const double t =
+          fm.fixed + (double)rounds * (fm.round + (double)split_stages[ks] * (fm.stage + fm.load * busy)) + reduce;
       if (t < limit) {
         limit = t;
-        best = Fp8MidPlan{true, kForms[f].mt, kForms[f].wn, kForms[f].ring, (int)ks, need};
+        best = Fp8MidPlan{true, fm.mt, fm.wn, fm.ring, (int)ks, need};
       }
     }
   }
