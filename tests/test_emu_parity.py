@@ -67,6 +67,7 @@ test_k_tiles_per_wave = w4.test_k_tiles_per_wave
 test_k_stationary_split_sums = w4.test_k_stationary_split_sums
 test_a_scale_that_is_not_finite_stays_in_its_column = w4.test_a_scale_that_is_not_finite_stays_in_its_column
 test_scales_near_the_end_of_the_bf16_range = w4.test_scales_near_the_end_of_the_bf16_range
+test_decode_of_tiny_and_huge_activations = w4.test_decode_of_tiny_and_huge_activations
 test_decode_sums_round_to_the_exact_result = w4.test_decode_sums_round_to_the_exact_result
 test_k_phases_inside_the_workgroup = w4.test_k_phases_inside_the_workgroup
 

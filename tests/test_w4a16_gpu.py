@@ -176,6 +176,21 @@ def test_scales_near_the_end_of_the_bf16_range(gpu, form):
     orc.assert_parity(got * np.float32(1e-36), case.oracle() * np.float32(1e-36), f"scales of 1e36, {form}")
 
 
+@pytest.mark.parametrize("form", _DECODE_FORMS)
+@pytest.mark.parametrize("dtype,size", [("f16", 2e-5), ("f16", 1.5e4), ("bf16", 1e-30), ("bf16", 1e30)])
+def test_decode_of_tiny_and_huge_activations(gpu, form, dtype, size):
+    """Activations at both ends of the range (fp16: subnormal, and sums over a group of 64 beyond 65504), scales that bring the
+    results back to the middle: the pieces that row sums are split into hold all of them."""
+    M, K, g, env = _DECODE_FORMS[form]
+    rng = np.random.default_rng(1490 + M)
+    act = (size * (1 + 0.3 * rng.standard_normal((M, K)))).astype(np.float32)
+    sv = (0.02 / np.float64(size) * (1 + 0.2 * rng.random((K // g, 336)))).clip(1e-4 if dtype == "f16" else 1e-38, 1e38)
+    case = W4Case(1491, M, K, 336, g=g, kind="awq", dtype=dtype, scales=sv.astype(np.float32), act=act)
+    with _env(**env):
+        got = W4Device(case, gpu).gemm_f32()
+    orc.assert_parity(got, case.oracle(), f"activations of {size:g} {dtype} {form}")
+
+
 @pytest.mark.parametrize("form", ["start_1", "start_2", "start_2_eight", "start_4"])
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_decode_sums_round_to_the_exact_result(gpu, form, dtype):
@@ -268,8 +283,8 @@ def test_prefill_bf16_long_rows(gpu, K):
     ("bf16", "gptq", 64, 96, 128, 256),    # a single k tile
 ])
 def test_prefill_row_tiles(gpu, rows, nt, dtype, kind, g, M, K, N):
-    """The large-M path with 64-row (1, 2 or 4 column tiles per wave) and 128-row workgroup tiles, whichever the
-    planner would pick."""
+    """The prefill kernel in blocks of 64 rows (1, 2 or 4 column tiles per wave) and of 128, whichever the planner
+    would pick."""
     case = W4Case(1260 + rows + M, M, K, N, g=g, kind=kind, dtype=dtype)
     dev = W4Device(case, gpu)
     with _env(KSQ_W4_PREFILL_ROWS=rows, KSQ_W4_PREFILL_NT=nt):
@@ -363,7 +378,7 @@ def test_prefill_128_rows_split_k(gpu, ksplit, waves, kg, ct, dtype, kind, g, M,
     ("bf16", "gptq", 64, 512, 1024, 256),
 ])
 def test_prefill_split_k(gpu, ksplit, nt, dtype, kind, g, M, K, N):
-    """The 64-row large-M kernel with K split over workgroups (fp32 partial tiles through the workspace, summed in split
+    """The prefill kernel in blocks of 64 rows with K split over workgroups (fp32 partial tiles through the workspace, summed in split
     order by a second kernel): parity, bit-identical repeats, and the fall-back to one split when the workspace holds
     nothing beyond the bf16 front part."""
     from ksanallm_amd import capi
@@ -438,12 +453,12 @@ def test_accumulator_stationary_split_k(gpu, lds, ksplit, dtype, kind, g, M, K, 
     ("bf16", "gptq", 64, 24, 10240, 272),    # 80 k tiles with two row tiles: split
     ("f16", "gptq", 128, 24, 2048, 4112),    # one column tile per CU and a bit: activations through registers
     ("bf16", "awq", 128, 64, 1152, 16400),   # four tiles per workgroup: activations through LDS, bf16 with CNT = 4
-    ("f16", "awq", 128, 100, 12288, 528),    # M >= 65, K >= 96 M: the 64-row kernel with K split in two
+    ("f16", "awq", 128, 100, 12288, 528),    # M >= 65, a long K: the prefill kernel with K split
     ("bf16", "gptq", 128, 128, 12288, 272),
 ])
 def test_planner_choices_without_overrides(gpu, dtype, kind, g, M, K, N):
     """Shapes picked so that the launch planners, left alone, take the split-K and LDS forms of the kernels for
-    17 <= M <= 64 and the split-K form of the 64-row large-M kernel; twice, bit for bit, and without a workspace."""
+    17 <= M <= 64 and the split-K form of the prefill kernel; twice, bit for bit, and without a workspace."""
     case = W4Case(1400 + M + N, M, K, N, g=g, kind=kind, dtype=dtype)
     dev = W4Device(case, gpu)
     got1 = dev.gemm_f32()
@@ -534,7 +549,7 @@ def test_prefill_bf16_row_magnitudes(gpu):
 @pytest.mark.parametrize("M", [16, 65, 600])
 def test_bf16_scales_far_outside_the_fp16_range(gpu, M):
     """bf16 group scales from 1e-6 to 1e5, different per column block and with a wide spread inside some columns: the
-    decode kernels (M = 16) keep scales in fp32, the 64-row and 128-row kernels (M = 65, 600) run their matrix
+    decode kernels (M = 16) keep scales in fp32, the prefill kernel (M = 65, 600) runs its matrix
     instructions in fp16 and must still be right, column block by column block."""
     K, N = 1024, 1024
     rng = np.random.default_rng(1290 + M)
@@ -675,8 +690,8 @@ def test_config2_awq_bf16_prefill_rows_subset(gpu, K, N):
 @pytest.mark.parametrize("K,N", [(8192, 8192), (28672, 8192)])
 def test_config3_gptq_70b_rows_subset(gpu, K, N):
     """The o and down projections of Llama-2-70B at M = 32, 64 and 256 through the product path: these
-    are the shapes where the planners split K over workgroups for 17 <= M <= 64 and (down, M = 256) in the 64-row
-    large-M kernel.  The oracle checks a seeded subset of rows."""
+    are the shapes where the planners split K over workgroups for 17 <= M <= 64 and (down, M = 256) in the
+    prefill kernel.  The oracle checks a seeded subset of rows."""
     import torch
 
     case = W4Case(3000 + K + N, 256, K, N, kind="gptq", dtype="f16")
