@@ -140,22 +140,23 @@ def test_config2_prefill_all_shapes(gpu, name, K, N, dtype):
     torch.cuda.empty_cache()
 
 
-def test_64_row_kernel_more_than_eight_row_blocks(gpu):
-    """A shape the planner gives to the 64-row kernel with more than eight row blocks, so that the workgroup order
-    walks several super-tile rows."""
+def test_more_than_eight_blocks_of_64_rows(gpu):
+    """A shape that the planner covers with nine and sixteen blocks of 64 rows, so that the workgroup order walks
+    several bands of eight row blocks."""
     import torch
 
     w = BigW4(torch, gpu, 2200, 2048, 1024, "awq", "f16")
     for M in (576, 1000):
-        w.check(M, what=f"64-row M={M}")
+        w.check(M, what=f"blocks of 64 rows M={M}")
 
 
 @pytest.mark.parametrize("kind,dtype,K,N", [("awq", "bf16", 4096, 22016), ("awq", "f16", 4096, 22016),
                                             ("gptq", "f16", 28672, 8192)])
 def test_wide_shapes_33_to_64_rows(gpu, kind, dtype, K, N):
     """33 to 64 rows on shapes whose columns fill the device several times over (or fill it, with a K long enough to
-    split) go through the 64-row kernel of the large-M path, 32 rows and fewer through the decode kernels: both sides
-    of that boundary, ragged row counts, bf16 (re-encoded activations) and fp16, and the K split."""
+    split) go through the prefill kernel in one block of 64 rows -- bf16 with K below 6144, and the long K, from 49
+    rows -- and fewer rows through the decode kernels: both sides of that boundary, ragged row counts, bf16 (re-encoded
+    activations) and fp16, and the K split."""
     import torch
 
     w = BigW4(torch, gpu, 2300 + K + N, K, N, kind, dtype)
